@@ -87,6 +87,12 @@ int qvex_qmv_w4g64_mfma(const uint16_t* x, const uint32_t* w, const uint16_t* sc
 int qvex_qmv_affine(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
                     const uint16_t* biases, uint16_t* y, int M, int N, int K, int bits,
                     int group_size, void* stream);
+/* The same product for any M >= 1 (prompt chunks) on the matrix cores, from the
+ * same layout: sum q*x and sum x per group in fp32, folded with the group's
+ * scale and bias, one bf16 rounding. A row's result does not depend on M. */
+int qvex_affine_gemm(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
+                     const uint16_t* biases, uint16_t* y, int M, int N, int K, int bits,
+                     int group_size, void* stream);
 /* out[l, :] = bf16(s * q + b) of row ids[l] (clamped to [0, V)): mx.dequantize
  * of the gathered rows in QEmbedding.__call__ (engine/model.py:126-130).
  * H % group_size == 0; w, out 16-byte aligned. */

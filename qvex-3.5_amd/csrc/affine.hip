@@ -8,7 +8,7 @@
 // row of K codes is K*bits/32 words. Per (row, group): a bf16 scale s and bias
 // b, w = s*q + b.
 //
-// Three kernels:
+// Four kernels:
 //   * qmv_affine_kernel: y = x W^T for 1..8 activation rows, VALU only. A chunk
 //     is 32 consecutive codes of one row = `bits` words (K % 32 == 0 and the
 //     group is a multiple of 32, so a chunk lies in one group). Each lane
@@ -17,6 +17,8 @@
 //     words), then accumulates d = sum q*x and X = sum x per activation row in
 //     fp32 and folds acc += s*d + b*X. R weight rows per wave share the
 //     activation chunk; lanes stride over the chunks; one wave sum per output.
+//   * affine_gemm_kernel: the same product for any number of rows (prompt
+//     chunks) on the matrix cores.
 //   * embed_affine_kernel: the rows of an embedding table, bf16(s*q + b).
 //   * widen_w4_kernel: lossless re-encoding of a width <= 4, group % 64 == 0
 //     weight as 4-bit group-64 (codes widened to nibbles, a group-128 scale and
@@ -60,6 +62,7 @@ __device__ __forceinline__ void load_chunk(const uint32_t* __restrict__ p, uint3
 }
 
 constexpr int AFF_MAXM = 8;    // activation rows per launch
+constexpr long AFF_GEMM_TALL = 512;    // blocks of 64 rows from which the GEMM takes them
 
 // AFF_R weight rows per wave share each activation chunk: 1 for one or two
 // activation rows (81 VGPRs, more waves in flight: 12.6 against 13.6 us for a
@@ -143,6 +146,212 @@ __global__ __launch_bounds__(256) void qmv_affine_kernel(const uint16_t* __restr
         if (m < M) y[(size_t)m * N + row] = f32_to_bf16(acc[r][m]);
     }
   }
+}
+
+// ---------------------------------------------------------------- prompt chunks
+//
+// y = x W^T on the matrix cores without rounding a weight: the codes themselves
+// are bf16 numbers (integers up to 255 are exact), so a group's d = sum q*x comes
+// from MFMAs on the raw codes, X = sum x from an MFMA against ones (it lands in
+// d's lanes), both in fp32, and acc += s*d + b*X folds the group as the VALU
+// kernel does. A row's order of sums depends on neither M nor the block shape.
+//
+// A block is 4 waves, 16 MT rows x 64 outputs, one 16-output tile per wave; a
+// stage of the k loop is 128 codes (4 MFMA steps of 32). Activations go through
+// LDS (16-byte chunk ch of a row at ch ^ row_swizzle(row): the 16 lanes of one
+// pass of a 16-byte read hit 16 bank groups). A wave's weights go through LDS of
+// its own: whole 16 BITS-byte row pieces by 16-byte loads, then BITS bytes (8
+// codes) per lane and step. (Taken from global memory by the lanes that use them,
+// 8 bytes of each of 16 rows per load, a stage cost about 1 us whatever MT.)
+// (scale, bias) pairs: one load per lane serves four stages, broadcast by a lane
+// permute per group. Bound by issue: a step's extraction (12 VALU instructions
+// for 8 bits), 8 fmas per row tile and group, 2 MFMAs per row tile.
+// us, against chunks of 8 rows through the VALU kernel: 200 rows of 4096 x 4096 at
+// 8 bits 34 (368), 512 rows of 12288 x 4096 at 6 bits 158, 1024 rows of
+// 24576 x 4096 at 8 bits 506.
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ int row_swizzle(int r) {
+  const int b = (r >> 2) & 3;                                   // b -> 0, 2, 3, 1
+  return ((((b << 1) & 3) ^ ((b >> 1) * 3)) << 2) | (r & 3);
+}
+
+// the 8 codes at bit `sh` (a multiple of 8) of the words (lo, hi), as bf16
+template <int BITS>
+__device__ __forceinline__ bf16x8_t codes8(uint32_t lo, uint32_t hi, int sh) {
+  constexpr uint32_t mask = (1u << BITS) - 1u;
+  uint32_t v[2] = {lo, hi};
+  if constexpr (BITS != 4 && BITS != 8) {
+    v[0] = __builtin_amdgcn_alignbit(hi, lo, sh);
+    v[1] = hi >> sh;
+  }
+  float f[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int o = j * BITS, wi = o >> 5, s = o & 31;
+    const uint32_t q = s + BITS <= 32 ? v[wi] >> s : __builtin_amdgcn_alignbit(v[1], v[0], s);
+    f[j] = (float)(q & mask);
+  }
+  u32x4 r;      // the high halves: exact
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    r[j] = __builtin_amdgcn_perm(__float_as_uint(f[2 * j + 1]), __float_as_uint(f[2 * j]), 0x07060302u);
+  return __builtin_bit_cast(bf16x8_t, r);
+}
+
+template <int BITS, int G32, int MT>     // G32: 32-code steps per group
+__global__ __launch_bounds__(256) void affine_gemm_kernel(const uint16_t* __restrict__ x,
+                                                          const uint32_t* __restrict__ w,
+                                                          const uint16_t* __restrict__ scales,
+                                                          const uint16_t* __restrict__ biases,
+                                                          uint16_t* __restrict__ y, int M, int N, int K) {
+  constexpr int NG = 4 / G32;                      // groups per stage, and of four stages per lane
+  constexpr int NW = (16 * BITS + 63) / 64;        // 16-byte weight loads per lane and stage
+  constexpr int PITCH = 16 * BITS + 16;            // bytes of a weight row of one stage in LDS
+  __shared__ u32x4 xs[2][MT * 256];
+  __shared__ __align__(16) uint8_t ws[2][4][16 * PITCH];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane >> 4, i16 = lane & 15;
+  // consecutive blocks of one XCD (dispatch is round-robin over 8) share their weights
+  const int row_blocks = (M + 16 * MT - 1) / (16 * MT), columns = (N + 63) / 64;
+  const int at = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
+  const int column = at / row_blocks, m0 = (at - column * row_blocks) * 16 * MT;
+  if (column >= columns) return;
+  const int n0 = column * 64 + wave * 16, n = n0 + i16;
+  const int chunks = K >> 5, groups = chunks / G32, stages = (chunks + 3) >> 2;
+  const int words = chunks * BITS;                 // of a weight row
+
+  struct Stage {
+    u32x4 x[MT], w[NW];
+  };
+  const uint16_t* xp[MT];
+  int xl[MT], wl[NW], wo[NW];
+  const uint32_t* wp[NW];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int row = (tid >> 4) + 16 * i;
+    xp[i] = x + (size_t)min(m0 + row, M - 1) * K;
+    xl[i] = row * 16 + ((tid & 15) ^ row_swizzle(row));
+  }
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {                   // 16 rows x BITS pieces; rows past N repeat the last
+    const int id = min(lane + 64 * i, 16 * BITS - 1), row = id / BITS, piece = id - row * BITS;
+    wp[i] = w + (size_t)min(n0 + row, N - 1) * words;
+    wo[i] = 4 * piece;
+    wl[i] = row * PITCH + 16 * piece;
+  }
+  // stages past the last repeat it; what lies past K is never used
+  auto load = [&](Stage& t, int st) __attribute__((always_inline)) {
+    st = min(st, stages - 1);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) t.x[i] = load16(xp[i] + min(st * 128 + (tid & 15) * 8, K - 8));
+    if (G32 == 4 || st * 4 + 4 <= chunks) {
+#pragma unroll
+      for (int i = 0; i < NW; ++i) t.w[i] = *reinterpret_cast<const u32x4_a4*>(wp[i] + st * 4 * BITS + wo[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NW; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t.w[i][e] = wp[i][min(st * 4 * BITS + wo[i] + e, words - 1)];
+    }
+  };
+  auto stage_to_lds = [&](const Stage& t, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) xs[buf][xl[i]] = t.x[i];
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+      if (16 * BITS % 64 == 0 || lane + 64 * i < 16 * BITS) *reinterpret_cast<u32x4*>(&ws[buf][wave][wl[i]]) = t.w[i];
+  };
+  // (scale, bias) of four stages: lane (c, i) holds row i's groups NG c .. NG c + NG - 1 of the 4 NG
+  const uint16_t* sr = scales + (size_t)min(n, N - 1) * groups;
+  const uint16_t* br = biases + (size_t)min(n, N - 1) * groups;
+  auto load_scales = [&](uint32_t (&sb)[NG], int st0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const int at_g = min(st0 * NG + NG * c + g, groups - 1);
+      sb[g] = (uint32_t)sr[at_g] | (uint32_t)br[at_g] << 16;
+    }
+  };
+
+  f32x4_t acc[MT], d[MT], X[MT];
+  const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) acc[mt] = d[mt] = X[mt] = zero;
+  const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+  const int a_at = i16 * 16, swz = row_swizzle(i16), w_at = i16 * PITCH + ((c * BITS) >> 2) * 4;
+  const int sh = ((c * BITS) & 3) * 8;
+  // step j of a stage, u its place among the four that sb covers
+  auto step = [&](int buf, int j, const uint32_t (&sb)[NG], int u) __attribute__((always_inline)) {
+    // a lane's 8 codes: BITS bytes, at most two words (the row's padding follows the last piece)
+    const uint8_t* from = &ws[buf][wave][w_at + j * 4 * BITS];
+    uint32_t lo, hi = 0;
+    if constexpr (BITS == 8) {
+      const u32x2 v = *reinterpret_cast<const u32x2*>(from);
+      lo = v.x;
+      hi = v.y;
+    } else {
+      lo = reinterpret_cast<const uint32_t*>(from)[0];
+      if constexpr (BITS != 2 && BITS != 4) hi = reinterpret_cast<const uint32_t*>(from)[1];
+    }
+    const bf16x8_t q = codes8<BITS>(lo, hi, sh);
+    const bool first = j % G32 == 0, last = j % G32 == G32 - 1;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const bf16x8_t a = __builtin_bit_cast(bf16x8_t, xs[buf][mt * 256 + a_at + ((4 * j + c) ^ swz)]);
+      d[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, q, first ? zero : d[mt], 0, 0, 0);
+      X[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ones, first ? zero : X[mt], 0, 0, 0);
+    }
+    if (!last) return;
+    const uint32_t v = (uint32_t)__shfl((int)sb[j / G32], 16 * u + i16, 64);   // group NG u + j / G32
+    const float s = bf16_lo(v), b = bf16_hi(v);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[mt][r] = fmaf(s, d[mt][r], fmaf(b, X[mt][r], acc[mt][r]));
+  };
+
+  // stage st is computed from LDS, st + 1 and st + 2 are in registers or on their way
+  Stage t[2];
+  uint32_t sb[NG], sb_next[NG];
+  load(t[0], 0);
+  load_scales(sb, 0);
+  load(t[1], 1);
+  stage_to_lds(t[0], 0);
+  load(t[0], 2);
+  __syncthreads();
+#pragma unroll 1
+  for (int st0 = 0; st0 < stages; st0 += 4) {
+    load_scales(sb_next, min(st0 + 4, stages - 1));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int st = st0 + u, buf = u & 1;
+      if (st >= stages) break;
+      const int steps = chunks - st * 4;
+      if (G32 == 4 || steps >= 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) step(buf, j, sb, u);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (j < steps) step(buf, j, sb, u);
+      }
+      stage_to_lds(t[buf ^ 1], buf ^ 1);
+      load(t[buf ^ 1], st + 3);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) sb[g] = sb_next[g];
+  }
+
+  if (n >= N) return;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + 16 * mt + 4 * c + r;
+      if (m < M) y[(size_t)m * N + n] = f32_to_bf16(acc[mt][r]);
+    }
 }
 
 // One block per gathered row; a thread per 32-code chunk writes 64 bytes.
@@ -245,6 +454,34 @@ void launch_qmv(hipStream_t st, const uint16_t* x, const uint32_t* w, const uint
                        M, N, K, gs);
 }
 
+template <int BITS, int G32>
+void launch_gemm_group(hipStream_t st, const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
+                       uint16_t* y, int M, int N, int K) {
+  const long columns = (N + 63) / 64;
+  auto go = [&](auto kernel, int rows) {
+    const long blocks = columns * ((M + rows - 1) / rows);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((blocks + 7) / 8 * 8)), dim3(256), 0, st, x, w, s, b, y, M, N, K);
+  };
+  // Tall blocks extract each code for more rows; below AFF_GEMM_TALL of them the
+  // chip is not full and shorter ones finish sooner (us, 8 bits, K = 4096, blocks of
+  // 64 | 32 rows: 64 x 4096 33 | 24, 200 x 4096 37 | 34, 512 x 4096 51 | 64,
+  // 100 x 24576 65 | 86; 20 x 24576 at 5 bits, half of 64 rows empty, 49 | 38)
+  if (M <= 16)
+    go(affine_gemm_kernel<BITS, G32, 1>, 16);
+  else if (M <= 32 || columns * ((M + 63) / 64) < AFF_GEMM_TALL)
+    go(affine_gemm_kernel<BITS, G32, 2>, 32);
+  else
+    go(affine_gemm_kernel<BITS, G32, 4>, 64);
+}
+
+template <int BITS>
+void launch_affine_gemm(hipStream_t st, const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
+                        uint16_t* y, int M, int N, int K, int gs) {
+  if (gs == 5) launch_gemm_group<BITS, 1>(st, x, w, s, b, y, M, N, K);
+  if (gs == 6) launch_gemm_group<BITS, 2>(st, x, w, s, b, y, M, N, K);
+  if (gs == 7) launch_gemm_group<BITS, 4>(st, x, w, s, b, y, M, N, K);
+}
+
 template <int BITS>
 void launch_embed(dim3 grid, hipStream_t st, const int32_t* ids, const uint32_t* w, const uint16_t* s,
                   const uint16_t* b, uint16_t* out, int V, int H, int gs) {
@@ -271,6 +508,21 @@ extern "C" int qvex_qmv_affine(const uint16_t* x, const uint32_t* w, const uint1
   QVEX_CHECK_ARG(qvex_aligned(x, 16) && qvex_aligned(w, 16), "qvex_qmv_affine: x and w must be 16-byte aligned");
   AFFINE_BITS_SWITCH(bits, launch_qmv, (hipStream_t)stream, x, w, scales, biases, y, M, N, K, gs);
   QVEX_CHECK_LAUNCH("qvex_qmv_affine");
+  return QVEX_OK;
+}
+
+extern "C" int qvex_affine_gemm(const uint16_t* x, const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
+                                uint16_t* y, int M, int N, int K, int bits, int group_size, void* stream) {
+  QVEX_CHECK_ARG(x && w && scales && biases && y, "qvex_affine_gemm: null pointer");
+  const int gs = group_shift(group_size);
+  QVEX_CHECK_ARG(width_ok(bits) && gs > 0, "qvex_affine_gemm: bits=%d group_size=%d (bits 2,3,4,5,6,8; groups 32,64,128)",
+                 bits, group_size);
+  QVEX_CHECK_ARG(M >= 1 && N >= 1 && K >= group_size && K % group_size == 0,
+                 "qvex_affine_gemm: M=%d N=%d K=%d (K a positive multiple of the group size %d)", M, N, K, group_size);
+  QVEX_CHECK_ARG(((M + 15L) / 16) * ((N + 63L) / 64) <= (1L << 30), "qvex_affine_gemm: M=%d N=%d too large", M, N);
+  QVEX_CHECK_ARG(qvex_aligned(x, 16) && qvex_aligned(w, 16), "qvex_affine_gemm: x and w must be 16-byte aligned");
+  AFFINE_BITS_SWITCH(bits, launch_affine_gemm, (hipStream_t)stream, x, w, scales, biases, y, M, N, K, gs);
+  QVEX_CHECK_LAUNCH("qvex_affine_gemm");
   return QVEX_OK;
 }
 

@@ -25,6 +25,7 @@ SIGNATURES: dict[str, list] = {
     "qvex_read_probe": [P, U64, P, I, I, I, P],
     "qvex_qmv_w4g64_mfma": [P, P, P, P, P, I, I, I, I, I, P],
     "qvex_qmv_affine": [P, P, P, P, P, I, I, I, I, I, P],
+    "qvex_affine_gemm": [P, P, P, P, P, I, I, I, I, I, P],
     "qvex_embed_affine": [P, I, P, P, P, I, I, I, I, P, P],
     "qvex_affine_widen_w4g64": [P, P, P, I, I, I, I, P, P, P, P],
     "qvex_w4g64_pack": [P, P, P, I, I, P, U64, P],

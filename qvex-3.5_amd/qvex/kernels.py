@@ -93,9 +93,11 @@ def _check_affine(w, scales, biases, K: int, group_size: int, bits: int):
 
 
 def quantized_matmul_affine(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
-                            group_size: int, bits: int, out: torch.Tensor | None = None) -> torch.Tensor:
+                            group_size: int, bits: int, out: torch.Tensor | None = None,
+                            gemm: bool = False) -> torch.Tensor:
     """y = x @ dequant(w)^T for any supported width (qvex_qmv_affine); x at most
-    8 rows, w int32 [N, K*bits/32], scales/biases bf16 [N, K/group_size]."""
+    8 rows, w int32 [N, K*bits/32], scales/biases bf16 [N, K/group_size]. gemm:
+    any number of rows, on the matrix cores (qvex_affine_gemm)."""
     K = x.shape[-1]
     x2 = x.reshape(-1, K)
     M = x2.shape[0]
@@ -107,7 +109,7 @@ def quantized_matmul_affine(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
     _check(out, "out", torch.bfloat16)
     if out.numel() != M * N:
         raise _C.QvexError("out has the wrong size")
-    _C.call("qvex_qmv_affine", _ptr(x2), _ptr(w), _ptr(scales), _ptr(biases), _ptr(out), M, N, K, bits,
+    _C.call("qvex_affine_gemm" if gemm else "qvex_qmv_affine", _ptr(x2), _ptr(w), _ptr(scales), _ptr(biases), _ptr(out), M, N, K, bits,
             group_size, _stream())
     return out
 

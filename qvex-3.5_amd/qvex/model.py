@@ -140,7 +140,8 @@ class QLinear:
     losslessly as 4-bit group-64 (bits <= 4, group 64 or 128: every 3-bit layer
     of a mixed 4/3-bit model) is widened once, at construction, and then takes
     every path below exactly as a 4-bit layer does; the other widths run the
-    any-width VALU product (qvex_qmv_affine) in chunks of 8 rows, without the
+    any-width VALU product (qvex_qmv_affine) on up to 8 rows and in chunks of 8
+    below DENSE_MIN_ROWS, the any-width MFMA GEMM (qvex_affine_gemm) above, without the
     fused epilogues. For the 4-bit group-64 layout: when K is
     a multiple of 256 the layer also keeps the tile-packed copy (pack_w4), built
     once here, and runs every call of 1..8 rows - decode, MTP drafts, verify of
@@ -149,7 +150,8 @@ class QLinear:
     number of rows. Calls of 9..DENSE_MIN_ROWS-1 rows (short prefill tails) run
     it on chunks of 8 rows, so their rows have the same bits too; longer calls (prefill) run the packed
     MFMA GEMM (weights dequantized to bf16 in registers). Without a packed copy
-    (K not a multiple of 256) the MLX-layout kernel takes chunks of 8 rows."""
+    (K not a multiple of 256) the MLX-layout kernel takes calls, and chunks of
+    short tails, of 8 rows, and longer calls run qvex_affine_gemm."""
 
     PACKED_MAX_ROWS = 8
     # calls of at least this many rows (prefill) run the packed GEMM; 0 disables it
@@ -256,6 +258,9 @@ class QLinear:
             kernels.packed_gemm(x2.contiguous(), self.packed, self.N, out=o2)
             return out.view(*lead, self.N)
         w, sc, bi = self._mlx_on(x.device)
+        if self.packed is None and self.DENSE_MIN_ROWS and M >= max(self.DENSE_MIN_ROWS, QMV_MAX_ROWS + 1):
+            kernels.quantized_matmul_affine(x2, w, sc, bi, self.group_size, self.bits, out=o2, gemm=True)
+            return out.view(*lead, self.N)
         for m0 in range(0, M, QMV_MAX_ROWS):
             m1 = min(M, m0 + QMV_MAX_ROWS)
             kernels.quantized_matmul(x2[m0:m1], w, sc, bi, out=o2[m0:m1], group_size=self.group_size,
