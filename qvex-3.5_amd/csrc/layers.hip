@@ -10,6 +10,7 @@
 // [Hkv, cap, D] bf16 per layer (one contiguous key run per kv head); the
 // GDN conv input window [3 + T, C] is kept per call so that the conv state
 // after L accepted tokens is rows L..L+2 of it (a pointer pick on rollback).
+#include "attn_prefill.h"
 #include "qvex_common.h"
 #include "rms_row.h"
 
@@ -1155,6 +1156,12 @@ extern "C" int qvex_attention(const uint16_t* q, const uint16_t* k_cache, const 
   QVEX_CHECK_ARG(ntile <= 65535 && nsplit <= 65535, "qvex_attention: grid too large");
   const float scale = 1.0f / sqrtf((float)D);
   hipStream_t st = (hipStream_t)stream;
+  if (ntile >= qvex::ATT_PREFILL_TILES) {
+    qvex::attention_prefill(q, k_cache, v_cache, pos0, L, Hq, Hkv, D, cap, ntile, nsplit, QT, keys_per_split, scale,
+                            gate, gate_stride, out, (float*)workspace, stream);
+    QVEX_CHECK_LAUNCH("qvex_attention/prefill");
+    return QVEX_OK;
+  }
   const dim3 pgrid(Hkv, ntile, nsplit);
   if (D == 256) {
     hipLaunchKernelGGL((attn_mfma_partial_kernel<256>), pgrid, dim3(256), 0, st, q, k_cache, v_cache, pos0, L, Hq,

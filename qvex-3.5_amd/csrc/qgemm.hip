@@ -46,6 +46,7 @@
 // buffers that these replace: 512 rows of 24576 x 4096 101 (255), 4096 x 12288 78
 // (195), 12352 x 4096 64 (156), 10240 x 4096 59 (138), 4096 x 4096 29 (67); 37 rows
 // of 10240 x 4096 15 (64).
+#include "lds_dma.h"
 #include "qvex_common.h"
 #include "w4_dequant.h"
 
@@ -59,31 +60,6 @@ constexpr int QG_WSLOT = 1024 + 256;        // a tile's codes and (scale, bias) 
 
 typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
-
-// One DMA of 16 (4) bytes per lane from global memory to LDS: lane l lands at
-// lds + 16 l (lds + 4 l). It has no register outputs; nothing reads the bytes
-// before the stage's vmcnt wait and barrier.
-__device__ __forceinline__ void dma16(uint32_t lds, uint32_t off, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-               : "memory", "m0");
-}
-__device__ __forceinline__ void dma16_nt(uint32_t lds, uint32_t off, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(off), "s"(base)
-               : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(uint32_t lds, uint32_t off, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base)
-               : "memory", "m0");
-}
-
-// At most N of this wave's DMAs still in flight, its LDS reads done, and every
-// wave of the block here. The builtin (LDS reads only) tells the compiler that
-// they are done: it would otherwise wait for them again behind later ones.
-template <int N>
-__device__ __forceinline__ void arrive() {
-  __builtin_amdgcn_s_waitcnt(0xc07f);
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
 
 __device__ __forceinline__ int row_swizzle(int r) {
   const int b = (r >> 2) & 3;                                   // b -> 0, 2, 3, 1
@@ -249,7 +225,7 @@ __global__ __launch_bounds__(64 * NW, PER_CU) void packed_gemm_kernel(const uint
   const int m0 = row * BM, tile0 = (column * NW + wave) * TPW;
   const int h_last = 2 * (K / QG_SET) - 1;
   Src src;
-  src.init(x, packed, (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds, M, K, m0, tile0, tiles, wave,
+  src.init(x, packed, lds_offset(lds), M, K, m0, tile0, tiles, wave,
            lane, h_last);
 
   f32x4_t acc[MT][TPW];
@@ -369,7 +345,7 @@ __global__ __launch_bounds__(256, 2) void packed_gemm_small_kernel(const uint16_
   const int tile = blockIdx.x * NW + wave;
   const int h_last = 2 * (K / QG_SET) - 1;
   Src src;
-  src.init(x, packed, (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds, M, K, 0, tile, tiles, wave,
+  src.init(x, packed, lds_offset(lds), M, K, 0, tile, tiles, wave,
            lane, h_last);
   f32x4_t acc[MT];
 #pragma unroll
