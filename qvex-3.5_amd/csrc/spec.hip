@@ -74,9 +74,16 @@ constexpr int NI = 8;   // float4 loads per thread per part
 // polynomial runs on the argument clamped to [-69, 88] (equal to x wherever its
 // value is used) and the out-of-range results are selected afterwards, so the
 // bits are those of the form that returns early (NaN gives 0 as there).
+// NONPOS: x <= 0 (or NaN), so nothing is to be done about the upper end. With the
+// scale as one shift-and-add, 19 VALU instructions instead of 24 per element of the
+// row statistics, which they bound beside HBM: 563 -> 516 us for 2304 rows of 248320.
+template <bool NONPOS = false>
 __device__ __forceinline__ float qx_expf(float x) {
-  const float xc = fminf(fmaxf(x, -69.0f), 88.0f);
-  const float n = rintf(xc * 1.44269504f);
+  const float xc = NONPOS ? fmaxf(x, -69.0f) : fminf(fmaxf(x, -69.0f), 88.0f);
+  // rint by adding 1.5 * 2^23 (the product is far below 2^22): the sum's low bits
+  // are n, so the scale by 2^n is one shift-and-add into the exponent below
+  const float sh = xc * 1.44269504f + 12582912.0f;
+  const float n = sh - 12582912.0f;
   float r = fmaf(n, -0.693145751953125f, xc);
   r = fmaf(n, -1.428606765330187e-06f, r);
   float p = 1.0f / 5040.0f;
@@ -87,9 +94,9 @@ __device__ __forceinline__ float qx_expf(float x) {
   p = fmaf(p, r, 0.5f);
   p = fmaf(p, r, 1.0f);
   p = fmaf(p, r, 1.0f);
-  const int e = (int)n;
-  const float v = p * __uint_as_float((uint32_t)(e + 127) << 23);
-  return x >= -69.0f ? (x > 88.0f ? __builtin_inff() : v) : 0.0f;
+  // p is in [0.7, 1.5] and n in [-100, 127]: a normal result, exactly p * 2^n
+  const float v = __uint_as_float(__float_as_uint(p) + (__float_as_uint(sh) << 23));
+  return x >= -69.0f ? (!NONPOS && x > 88.0f ? __builtin_inff() : v) : 0.0f;
 }
 
 __device__ __forceinline__ float wave_bfly_sum(float v) {
@@ -506,7 +513,7 @@ __device__ __forceinline__ void rowstats_block(const SpecArgs& a, int p, int row
     for (int it = 0; it < NI; ++it)
       if (ok[it]) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc = acc + qx_expf(z[it][e] - m);
+        for (int e = 0; e < 4; ++e) acc = acc + qx_expf<true>(z[it][e] - m);      // m is the part's maximum
       }
     const float s = block_sum(acc, red);
     if (t == 0) {
