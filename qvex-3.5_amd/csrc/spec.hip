@@ -76,7 +76,7 @@ constexpr int NI = 8;   // float4 loads per thread per part
 // bits are those of the form that returns early (NaN gives 0 as there).
 // NONPOS: x <= 0 (or NaN), so nothing is to be done about the upper end. With the
 // scale as one shift-and-add, 19 VALU instructions instead of 24 per element of the
-// row statistics, which they bound beside HBM: 563 -> 516 us for 2304 rows of 248320.
+// row statistics, which they bounded beside HBM: 563 -> 516 us for 2304 rows of 248320.
 template <bool NONPOS = false>
 __device__ __forceinline__ float qx_expf(float x) {
   const float xc = NONPOS ? fmaxf(x, -69.0f) : fminf(fmaxf(x, -69.0f), 88.0f);
@@ -421,7 +421,7 @@ __device__ __forceinline__ bool topk_thresh(const float (&zz)[4 * NI], const boo
 
 // Part p of row `row` (the block's work in spec_rowstats_kernel); zero_ctr:
 // this block clears the one-kernel finish counters (part 0 of row 0).
-template <bool BF>
+template <bool BF, bool LISTS = true>
 __device__ __forceinline__ void rowstats_block(const SpecArgs& a, int p, int row, bool zero_ctr) {
   __shared__ float red[4];
   __shared__ int redi[4];
@@ -499,7 +499,7 @@ __device__ __forceinline__ void rowstats_block(const SpecArgs& a, int p, int row
   // (m_p, S_p) of the part, which the unfiltered rules combine; the list form
   // without draft logits (the finish kernel) takes (c_0, S_p, cutoff) from the
   // lists alone, so its target rows skip the exponentials
-  if (!(a.fast && tgt && a.filt == 1)) {
+  if (!(LISTS && a.fast && tgt && a.filt == 1)) {
     float m = -__builtin_inff();
 #pragma unroll
     for (int it = 0; it < NI; ++it)
@@ -521,7 +521,7 @@ __device__ __forceinline__ void rowstats_block(const SpecArgs& a, int p, int row
       out[1] = s;
     }
   }
-  if (tgt && a.filt == 1) {
+  if (LISTS && tgt && a.filt == 1) {
     // this part's top_k largest z and the count of its values equal to the k-th
     __shared__ float lst[64];
     __shared__ __align__(16) float wl[4 * 64];
@@ -633,9 +633,20 @@ __device__ __forceinline__ void rowstats_block(const SpecArgs& a, int p, int row
   }
 }
 
-template <bool BF>
+// LISTS: the form with the top-k lists (filt == 1). Without them a thread holds its
+// 32 logits and little else: 54 registers instead of 172, 9 waves on a SIMD instead
+// of 2, and 2304 rows of 248320 fp32 logits take 354 us (6.5 TB/s) instead of 516.
+template <bool BF, bool LISTS>
 __global__ __launch_bounds__(NT) void spec_rowstats_kernel(SpecArgs a) {
-  rowstats_block<BF>(a, blockIdx.x, blockIdx.y, true);
+  rowstats_block<BF, LISTS>(a, blockIdx.x, blockIdx.y, true);
+}
+
+template <bool BF>
+void launch_rowstats(dim3 grid, hipStream_t st, const SpecArgs& a) {
+  if (a.filt == 1)
+    hipLaunchKernelGGL((spec_rowstats_kernel<BF, true>), grid, dim3(NT), 0, st, a);
+  else
+    hipLaunchKernelGGL((spec_rowstats_kernel<BF, false>), grid, dim3(NT), 0, st, a);
 }
 
 // ---------------------------------------------------------------- filter kernel (top-k / top-p)
@@ -982,13 +993,15 @@ struct WCtx {
   int n_extra;
 };
 
-__device__ __forceinline__ float weight(const WCtx& c, int j) {
-  const float z = pen_x(c.seen, c.pen, lg(c.tp, j, c.bf), j, c.extra, c.n_extra) * c.inv_temp;
-  const float ep = z >= c.cutoff ? qx_expf(z - c.mp) : 0.0f;
+// The weight of token j from its two logits (xq of a dense draft row only). mp and
+// mq are the rows' maxima, so both exponents are at most 0.
+__device__ __forceinline__ float weight_x(const WCtx& c, int j, float xt, float xq) {
+  const float z = pen_x(c.seen, c.pen, xt, j, c.extra, c.n_extra) * c.inv_temp;
+  const float ep = z >= c.cutoff ? qx_expf<true>(z - c.mp) : 0.0f;
   if (c.mode == 1) return ep;
   float eq, Sq;
   if (c.tq) {
-    eq = qx_expf(lg(c.tq, j, c.bf) * c.inv_temp - c.mq);
+    eq = qx_expf<true>(xq * c.inv_temp - c.mq);
     Sq = c.sq;
   } else {
     eq = (j == c.d) ? 1.0f : 0.0f;
@@ -998,6 +1011,49 @@ __device__ __forceinline__ float weight(const WCtx& c, int j) {
   const float t2 = eq * c.sp;
   const float r = t1 - t2;
   return r > 0.0f ? r : 0.0f;
+}
+
+__device__ __forceinline__ float weight(const WCtx& c, int j) {
+  return weight_x(c, j, lg(c.tp, j, c.bf), c.tq ? lg(c.tq, j, c.bf) : 0.0f);
+}
+
+// Logits j .. j + 3 of a row (j a multiple of 4; V is one too, so rows start
+// on a vector's boundary) as the statistics kernel reads them.
+__device__ __forceinline__ void lg4(const void* row, int j, int bf, float (&x)[4]) {
+  if (bf) {
+    const u32x2 v = __builtin_nontemporal_load(
+        reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(row) + j));
+    x[0] = bf16_lo(v.x);
+    x[1] = bf16_hi(v.x);
+    x[2] = bf16_lo(v.y);
+    x[3] = bf16_hi(v.y);
+  } else {
+    const u32x4 v = load_nt16(reinterpret_cast<const float*>(row) + j);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = __uint_as_float(v[e]);
+  }
+}
+
+// Sum of a thread's weights of part [base, end) in the fixed (it, e) order, both
+// rows requested before the first weight is formed.
+__device__ __forceinline__ float thread_weights(const WCtx& c, int base, int end) {
+  const int t = threadIdx.x;
+  float xt[NI][4], xq[NI][4];
+#pragma unroll
+  for (int it = 0; it < NI; ++it) lg4(c.tp, min(base + 4 * (t + NT * it), end - 4), c.bf, xt[it]);
+  if (c.tq) {
+#pragma unroll
+    for (int it = 0; it < NI; ++it) lg4(c.tq, min(base + 4 * (t + NT * it), end - 4), c.bf, xq[it]);
+  }
+  float acc = 0.0f;
+#pragma unroll
+  for (int it = 0; it < NI; ++it) {
+    const int j = base + 4 * (t + NT * it);
+    if (j >= end) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = acc + weight_x(c, j + e, xt[it][e], c.tq ? xq[it][e] : 0.0f);
+  }
+  return acc;
 }
 
 // weight() of a one-hot draft from the element's z (the value the statistics
@@ -1102,9 +1158,48 @@ __device__ __forceinline__ SpecWs spec_ws(const SpecArgs& a) {
   return w;
 }
 
+// The walk's weights as the step's decision record gives them.
+__device__ __forceinline__ WCtx decided(const SpecArgs& a, const SpecWs& W, int step) {
+  const int k = a.k;
+  const float* dd = W.dec + (long)step * 8;
+  const int n = __float_as_int(dd[0]);
+  WCtx c;
+  c.inv_temp = a.inv_temp;
+  c.tp = row_ptr(a, step, n);
+  c.bf = a.bf;
+  c.d = __float_as_int(dd[1]);
+  c.mp = dd[2]; c.sp = dd[3]; c.mq = dd[4]; c.sq = dd[5];
+  c.cutoff = dd[6];
+  c.seen = a.seen;
+  c.pen = a.pen;
+  c.extra = a.ids + (long)step * k;
+  c.n_extra = n;
+  c.tq = (n < k && a.draft) ? row_ptr(a, step, k + 1 + n) : nullptr;
+  c.mode = n < k ? 0 : 1;
+  return c;
+}
+
+// The thread and part sums of the sampling weights over part p.
+__device__ __forceinline__ void part_weights(const SpecArgs& a, const SpecWs& W, const WCtx& c, int p, int step,
+                                             float* red) {
+  const int base = p * PART, end = min(a.V, base + PART);
+  const float acc = thread_weights(c, base, end);
+  W.T[((long)step * a.P + p) * NT + threadIdx.x] = acc;
+  const float wp = block_sum(acc, red);
+  if (threadIdx.x == 0) W.W[(long)step * a.P + p] = wp;
+}
+
 // Kernel 2 (grid parts x steps): every block combines the step's row statistics
 // and runs the k accept tests (a few gathers), then block p makes the thread and
-// part sums of the sampling weights over part p of the sampling row.
+// part sums of the sampling weights over part p of the sampling row. With many
+// steps (DECIDE_STEPS) one block per step decides (WEIGHTS false, grid 1 x steps) and
+// spec_weights_kernel makes the sums: a decision is a chain of dependent loads of
+// about 5 us, which 31 parts x 256 steps of blocks repeated in several rounds.
+// 256 steps of 248320 logits with draft rows: 12 + 121 us (189 in one kernel, 205
+// with a load per logit); 128 steps 265 -> 241 in all, 16 to 32 no difference, fewer
+// a launch more.
+constexpr int DECIDE_STEPS = 32;
+template <bool WEIGHTS>
 __global__ __launch_bounds__(NT) void spec_decide_kernel(SpecArgs a) {
   __shared__ float rm[80], rs[80], rc[80];
   __shared__ float red[4];
@@ -1238,28 +1333,20 @@ __global__ __launch_bounds__(NT) void spec_decide_kernel(SpecArgs a) {
     c.mq = 0.0f;
     c.sq = 1.0f;
   }
-  const int base = p * PART, end = min(a.V, base + PART);
-  float acc = 0.0f;
-#pragma unroll
-  for (int it = 0; it < NI; ++it) {
-    const int j = base + 4 * (t + NT * it);
-    if (j < end) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc = acc + weight(c, j + e);
-    }
+  if (p == 0 && t == 0) {
+    float* dd = W.dec + (long)step * 8;
+    dd[0] = __int_as_float(n);
+    dd[1] = __int_as_float(c.d);
+    dd[2] = c.mp; dd[3] = c.sp; dd[4] = c.mq; dd[5] = c.sq;
+    dd[6] = c.cutoff;
   }
-  W.T[((long)step * a.P + p) * NT + t] = acc;
-  const float wp = block_sum(acc, red);
-  if (t == 0) {
-    W.W[(long)step * a.P + p] = wp;
-    if (p == 0) {
-      float* dd = W.dec + (long)step * 8;
-      dd[0] = __int_as_float(n);
-      dd[1] = __int_as_float(c.d);
-      dd[2] = c.mp; dd[3] = c.sp; dd[4] = c.mq; dd[5] = c.sq;
-      dd[6] = c.cutoff;
-    }
-  }
+  if constexpr (WEIGHTS) part_weights(a, W, c, p, step, red);
+}
+
+__global__ __launch_bounds__(NT) void spec_weights_kernel(SpecArgs a) {
+  __shared__ float red[4];
+  const SpecWs W = spec_ws(a);
+  part_weights(a, W, decided(a, W, blockIdx.y), blockIdx.x, blockIdx.y, red);
 }
 
 // Kernel 3 (one block per step): inverse-CDF walk over the stored part and
@@ -1275,21 +1362,7 @@ __global__ __launch_bounds__(NT) void spec_sample_kernel(SpecArgs a) {
   const int t = threadIdx.x;
   const int k = a.k;
   const SpecWs W = spec_ws(a);
-  const float* dd = W.dec + (long)step * 8;
-  const int n = __float_as_int(dd[0]);
-  WCtx c;
-  c.inv_temp = a.inv_temp;
-  c.tp = row_ptr(a, step, n);
-  c.bf = a.bf;
-  c.d = __float_as_int(dd[1]);
-  c.mp = dd[2]; c.sp = dd[3]; c.mq = dd[4]; c.sq = dd[5];
-  c.cutoff = dd[6];
-  c.seen = a.seen;
-  c.pen = a.pen;
-  c.extra = a.ids + (long)step * k;
-  c.n_extra = n;
-  c.tq = (n < k && a.draft) ? row_ptr(a, step, k + 1 + n) : nullptr;
-  c.mode = n < k ? 0 : 1;
+  WCtx c = decided(a, W, step);
   const float u = a.u_smp[step];
   // The walks are sequential fp32 sums (the fixed order), done by thread 0, but
   // over values the block first stages in LDS: the part sums, then the chosen
@@ -1419,7 +1492,7 @@ __global__ __launch_bounds__(NT) void spec_sample_kernel(SpecArgs a) {
     tok = sample_pass(c, a.V, a.P, u, Tpt, Wp, red);
   }
   if (t == 0) {
-    a.n_accept[step] = n;
+    a.n_accept[step] = c.n_extra;
     a.out_token[step] = tok;
   }
 }
@@ -2448,9 +2521,9 @@ static int spec_accept_impl(const void* target, const void* draft, int bf, const
              fast ? ncand : nullptr, fast ? ctr : nullptr, fast ? rres : nullptr};
   hipStream_t st = (hipStream_t)stream;
   if (a.bf)
-    hipLaunchKernelGGL(spec_rowstats_kernel<true>, dim3(P, S * rps), dim3(NT), 0, st, a);
+    launch_rowstats<true>(dim3(P, S * rps), st, a);
   else
-    hipLaunchKernelGGL(spec_rowstats_kernel<false>, dim3(P, S * rps), dim3(NT), 0, st, a);
+    launch_rowstats<false>(dim3(P, S * rps), st, a);
   QVEX_CHECK_LAUNCH("qvex_spec_accept/rowstats");
   if (fast) {
     hipLaunchKernelGGL(spec_finish_kernel, dim3(S * (k + 1)), dim3(NT), lds, st, a);
@@ -2464,9 +2537,16 @@ static int spec_accept_impl(const void* target, const void* draft, int bf, const
     hipLaunchKernelGGL(spec_wide_filter_kernel, dim3(S * (k + 1)), dim3(WT), 0, st, a);
     QVEX_CHECK_LAUNCH("qvex_spec_accept/wide_filter");
   }
-  hipLaunchKernelGGL(spec_decide_kernel, dim3(P, S), dim3(NT), 0, st, a);
+  if (greedy || S >= DECIDE_STEPS)
+    hipLaunchKernelGGL(spec_decide_kernel<false>, dim3(1, S), dim3(NT), 0, st, a);
+  else
+    hipLaunchKernelGGL(spec_decide_kernel<true>, dim3(P, S), dim3(NT), 0, st, a);
   QVEX_CHECK_LAUNCH("qvex_spec_accept/decide");
   if (!greedy) {
+    if (S >= DECIDE_STEPS) {
+      hipLaunchKernelGGL(spec_weights_kernel, dim3(P, S), dim3(NT), 0, st, a);
+      QVEX_CHECK_LAUNCH("qvex_spec_accept/weights");
+    }
     hipLaunchKernelGGL(spec_sample_kernel, dim3(S), dim3(NT), lds, st, a);
     QVEX_CHECK_LAUNCH("qvex_spec_accept/sample");
   }
@@ -2624,9 +2704,9 @@ extern "C" int qvex_sampler_scores(const void* logits, int logits_bf16, int R, i
   hipStream_t st = (hipStream_t)stream;
   if (!greedy) {
     if (a.bf)
-      hipLaunchKernelGGL(spec_rowstats_kernel<true>, dim3(P, R), dim3(NT), 0, st, a);
+      launch_rowstats<true>(dim3(P, R), st, a);
     else
-      hipLaunchKernelGGL(spec_rowstats_kernel<false>, dim3(P, R), dim3(NT), 0, st, a);
+      launch_rowstats<false>(dim3(P, R), st, a);
     QVEX_CHECK_LAUNCH("qvex_sampler_scores/rowstats");
     if (filt == 1) {
       hipLaunchKernelGGL(spec_filter_kernel, dim3(R), dim3(NT), 0, st, a);
