@@ -428,8 +428,8 @@ __global__ __launch_bounds__(256) void attn_mfma_partial_kernel(
   // K keys kb + 16h + li and V keys kb + 8lg .. +7 of a 128-key window (tiled
   // layouts above), issued together (keys past k_hi are masked out of the
   // softmax and get P = 0). The first window does not depend on the device
-  // position, so its loads go out before the position is read (this kernel runs
-  // the prefill, where the grid holds only visible splits).
+  // position, so its loads go out before the position is read (short prompt
+  // chunks run here too, on a grid of visible splits only; long ones in attn_prefill.hip).
   // A operand: Q row li, dims step*32 + 8*lg .. +7 (the 1/sqrt(D) scale is applied
   // to the scores). Requested first: loads complete in order, so the scores can
   // start once Q and K are in while the V columns still stream
