@@ -549,7 +549,12 @@ int qvex_attn_qk_rope(const uint16_t* proj, long p_stride, const uint16_t* q_nor
  * visible on every call: max_keys for a one-off call, the position at capture
  * for a captured graph) request their first keys before reading *pos0, the
  * others read it first and load nothing when past it; results do not depend on
- * known_keys. D is 128 or 256. workspace: qvex_attn_workspace_bytes(). */
+ * known_keys. D is 128 or 256.
+ * L >= 9 (prompt chunks): a row's sums restart every min(keys_per_split, 256) keys
+ * counted from key 0 whatever the call, so a row's bits do not depend on the chunk it
+ * comes in, nor on a keys_per_split of 256 or more; known_keys is not used.
+ * workspace: qvex_attn_workspace_bytes(), which never falls as L or max_keys grows
+ * (at one keys_per_split a workspace serves every smaller call too). */
 uint64_t qvex_attn_workspace_bytes(int L, int Hq, int Hkv, int D, int max_keys, int keys_per_split);
 int qvex_attention(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
                    const int32_t* pos0, int L, int Hq, int Hkv, int D, int cap, int max_keys,

@@ -428,8 +428,8 @@ __global__ __launch_bounds__(256) void attn_mfma_partial_kernel(
   // K keys kb + 16h + li and V keys kb + 8lg .. +7 of a 128-key window (tiled
   // layouts above), issued together (keys past k_hi are masked out of the
   // softmax and get P = 0). The first window does not depend on the device
-  // position, so its loads go out before the position is read (short prompt
-  // chunks run here too, on a grid of visible splits only; long ones in attn_prefill.hip).
+  // position, so its loads go out before the position is read (calls of 9 and
+  // more positions run in attn_prefill.hip).
   // A operand: Q row li, dims step*32 + 8*lg .. +7 (the 1/sqrt(D) scale is applied
   // to the scores). Requested first: loads complete in order, so the scores can
   // start once Q and K are in while the V columns still stream
@@ -1205,15 +1205,26 @@ extern "C" int qvex_attn_qk_rope(const uint16_t* proj, long p_stride, const uint
 namespace {
 constexpr int ATT_ROWS = 16;
 constexpr int ATT_DSPLIT = 4;   // combine blocks per row, each over D / 4 dims (4 x the blocks in flight)
+
 }
 
 extern "C" uint64_t qvex_attn_workspace_bytes(int L, int Hq, int Hkv, int D, int max_keys, int keys_per_split) {
-  if (L < 1 || Hkv < 1 || Hq % Hkv || keys_per_split < 1) return 0;
+  if (L < 1 || Hkv < 1 || Hq % Hkv || max_keys < 1 || keys_per_split < 1) return 0;
   const int GQ = Hq / Hkv;
   const int QT = ATT_ROWS / GQ < 1 ? 1 : ATT_ROWS / GQ;
   const int ntile = (L + QT - 1) / QT;
-  const int nsplit = (max_keys + keys_per_split - 1) / keys_per_split;
-  return (uint64_t)Hkv * ntile * nsplit * ATT_ROWS * (D + 2) * sizeof(float);
+  const bool prompt = L >= qvex::ATT_PROMPT_ROWS;
+  const uint64_t units = (max_keys - 1) / (prompt ? std::min(keys_per_split, qvex::ATT_UNIT) : keys_per_split) + 1;
+  uint64_t records = Hkv * ntile * units;
+  if (prompt) {
+    // a call of many blocks writes a record per group; what the smaller calls need (a
+    // record per unit) is covered too, so that a workspace serves every call up to its own
+    const uint64_t groups = Hkv * ntile * ((units - 1) / qvex::ATT_GROUP + 1);
+    const uint64_t small = Hkv * ((qvex::ATT_PROMPT_ROWS - 2) / QT + 1) * units;
+    const uint64_t one_unit = qvex::att_unit_blocks(D) * qvex::ATT_BLOCK_TILES;
+    records = std::min(records, std::max(std::max(groups, small), one_unit));
+  }
+  return records * ATT_ROWS * (D + 2) * sizeof(float);
 }
 
 extern "C" int qvex_attention(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
@@ -1233,12 +1244,16 @@ extern "C" int qvex_attention(const uint16_t* q, const uint16_t* k_cache, const 
   const int GQ = Hq / Hkv;
   const int QT = ATT_ROWS / GQ;
   const int ntile = (L + QT - 1) / QT;
-  const int nsplit = (max_keys + keys_per_split - 1) / keys_per_split;
+  const bool prompt = L >= qvex::ATT_PROMPT_ROWS;
+  const int unit = prompt ? std::min(keys_per_split, qvex::ATT_UNIT) : keys_per_split;
+  const int n = (max_keys - 1) / unit + 1;
+  const int units = prompt ? qvex::attention_units(Hkv, ntile, D, n) : 1;
+  const int nsplit = (n - 1) / units + 1;
   QVEX_CHECK_ARG(ntile <= 65535 && nsplit <= 65535, "qvex_attention: grid too large");
   const float scale = 1.0f / sqrtf((float)D);
   hipStream_t st = (hipStream_t)stream;
-  if (ntile >= qvex::ATT_PREFILL_TILES) {
-    qvex::attention_prefill(q, k_cache, v_cache, pos0, L, Hq, Hkv, D, cap, ntile, nsplit, QT, keys_per_split, scale,
+  if (prompt) {
+    qvex::attention_prefill(q, k_cache, v_cache, pos0, L, Hq, Hkv, D, cap, ntile, nsplit, QT, unit, units, scale,
                             gate, gate_stride, out, (float*)workspace, stream);
     QVEX_CHECK_LAUNCH("qvex_attention/prefill");
     return QVEX_OK;

@@ -666,21 +666,6 @@ class Attention:
         self.q_norm, self.k_norm = p["q_norm"], p["k_norm"]
         self._ws = None
 
-    def _prompt_kps(self, L, keys):
-        """Keys per split of a call of many rows. Long calls run blocks of 128 rows
-        (8 tiles of 16), two to a CU: the shortest splits whose blocks all fit at
-        once, and no more of them to write and merge (us for 512 rows, splits of
-        128 | 256 | 512 | 1024 | 2048: no earlier keys 27 | 32 | 41, 1024 54 | 45 | 46 | 70,
-        3584 153 | 87 | 68 | 74 | 123, 16384 638 | 431 | 308 | 223 | 204)."""
-        tiles = -(-L // max(1, 16 // (self.n_heads // self.n_kv)))
-        if tiles < 24:                   # a block per tile
-            return 512
-        blocks = self.n_kv * -(-tiles // 8)
-        kps = 128
-        while kps < 2048 and blocks * -(-keys // kps) > 512:
-            kps *= 2
-        return kps
-
     def _workspace(self, L, cap, kps, device):
         need = int(_C.lib().qvex_attn_workspace_bytes(L, self.n_heads, self.n_kv, self.head_dim, cap, kps))
         if self._ws is None or self._ws.numel() * 4 < need:
@@ -702,7 +687,9 @@ class Attention:
         pos = cache.counters.ptr(cache.index)
         # a captured call must work for every later context length: bound by capacity
         max_keys = cache.capacity if cache.counters.graph_mode else min(cache.capacity, cache.offset + L)
-        kps = self.decode_kps if L <= 8 else self._prompt_kps(L, max_keys)
+        # keys per 4-wave block: verify spreads ~ctx/32 waves per kv head; calls of more rows split at
+        # the kernel's own unit of keys, the same for every call
+        kps = self.decode_kps if L <= 8 else 512
         ws = self._workspace(L, max_keys, kps, x.device)
         o = torch.empty((L, H * D), dtype=torch.bfloat16, device=x.device)
         rot = cfg.rotary_dim

@@ -1,6 +1,7 @@
-"""qvex_attention on prompt chunks (calls of 24 or more 16-row tiles) against
-causal softmax attention times sigmoid(gate) in float64, at the edges of its
-128-row blocks, 32-key blocks and splits, and with the extremes of the scores.
+"""qvex_attention on prompt chunks (calls of 9 positions and more) against causal
+softmax attention times sigmoid(gate) in float64, at the edges of its 64-row
+blocks, 32-key blocks, units and groups of units, and with the extremes of the
+scores; a row's bits depend neither on the call nor on a keys_per_split of 256 or more.
 
 Bound: the output is rounded to bf16 (2^-8 |ref|), P is carried as two bf16 terms
 (2^-16 relative) and the sums are fp32: |err| <= 2^-8 |ref| + 2^-14 sigmoid(gate) sum p |v| + 1e-6."""
@@ -55,7 +56,12 @@ def reference(q, k, v, gate, pos0):
 @pytest.mark.parametrize("L,Hq,Hkv,D,pos0,kps,spare", [
     (93, 16, 4, 256, 0, 512, 0), (96, 16, 4, 256, 31, 128, 0), (97, 16, 4, 256, 995, 512, 0),
     (190, 4, 2, 128, 33, 128, 1), (130, 6, 2, 128, 257, 256, 0), (117, 6, 2, 256, 1, 512, 0),
-    (25, 16, 1, 128, 600, 128, 0), (370, 8, 8, 128, 5, 512, 1), (512, 16, 4, 256, 1536, 2048, 0)])
+    (25, 16, 1, 128, 600, 128, 0), (370, 8, 8, 128, 5, 512, 1), (512, 16, 4, 256, 1536, 2048, 0),
+    # 9 positions and up, one tile and part of a block
+    (9, 16, 4, 256, 119, 128, 0), (9, 2, 2, 128, 0, 256, 0), (17, 16, 16, 256, 255, 256, 0), (65, 4, 1, 256, 511, 256, 1),
+    # a group of four units per block: whole groups, a last one of one unit and of three, fewer than four units
+    (512, 8, 8, 256, 1600, 128, 0), (512, 8, 8, 256, 1900, 128, 1), (300, 8, 8, 256, 3700, 128, 0),
+    (520, 8, 8, 128, 3800, 128, 0), (2300, 16, 16, 256, 0, 1024, 0)])
 def test_prefill_attention(L, Hq, Hkv, D, pos0, kps, spare):
     q, k, v, gate = inputs(L, Hq, Hkv, D, pos0, seed=L + pos0)
     got = attention(q, k, v, gate, pos0, kps, spare).double()
@@ -93,3 +99,34 @@ def test_prefill_attention_nan_key_reaches_only_the_rows_that_see_it():
     assert got[50:, 4:8].all()
     got[50:, 4:8] = False
     assert not got.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,D,pos0,L,kps", [(16, 4, 256, 0, 90, 256), (16, 4, 256, 4000, 600, 256),
+                                                 (8, 8, 256, 2011, 512, 128), (8, 8, 128, 4001, 500, 128)])
+def test_prefill_attention_rows_over_block_forms(Hq, Hkv, D, pos0, L, kps):
+    """Parts that start inside a tile, a block of keys and a unit; the whole takes a
+    group of units per block (the last three), the parts one unit."""
+    q, k, v, gate = inputs(L, Hq, Hkv, D, pos0, seed=6, scale=4.0)
+    full = attention(q, k, v, gate, pos0, kps)
+    for lo, n in ((0, 9), (1, 16), (7, 33), (L - 70, 70)):
+        part = attention(q[lo:lo + n].contiguous(), k, v, gate[lo:lo + n].contiguous(), pos0 + lo, kps, spare=lo % 2)
+        assert torch.equal(part.view(torch.int16), full[lo:lo + n].view(torch.int16)), (lo, n)
+    if kps == 256:
+        assert torch.equal(attention(q, k, v, gate, pos0, 2048).view(torch.int16), full.view(torch.int16))
+
+
+def test_attention_workspace_serves_smaller_calls():
+    """The size never falls as a call grows, and a record per unit is its upper bound."""
+    size = _C.lib().qvex_attn_workspace_bytes
+    for Hq, Hkv, D in ((16, 4, 256), (8, 8, 128), (16, 1, 256), (8, 2, 128)):
+        QT = 16 // (Hq // Hkv)
+        for kps in (128, 256, 2048):
+            prev = {}
+            for L in (1, 8, 9, 17, 64, 100, 512, 1000):
+                last = 0
+                for keys in (1, 128, 129, 1000, 4096, 5000, 20000, 131072):
+                    n = int(size(L, Hq, Hkv, D, keys, kps))
+                    assert n >= last and n >= prev.get(keys, 0), (Hq, Hkv, D, kps, L, keys)
+                    assert n <= Hkv * -(-L // QT) * -(-keys // (kps if L < 9 else min(kps, 256))) * 16 * (D + 2) * 4
+                    prev[keys] = last = n
