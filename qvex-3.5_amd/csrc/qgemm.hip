@@ -24,7 +24,10 @@
 // Dequantization. A masked word is a pair of fp16 subnormals, codes at bits 0
 // and 16 (q * 2^-24) or at bits 4 and 20 (q * 2^-20): v_fma_mix_f32 reads either
 // half, so s * 2^24 (or 2^20) and b give s * q + b in one instruction per code
-// and 17 VALU instructions per 8 codes (27 with bf16 pairs unpacked to fp32).
+// and 17 VALU instructions per 8 codes (27 with bf16 pairs unpacked to fp32). Where
+// |s| is 2^104 or more s * 2^24 overflows and every sum it enters is infinite or NaN:
+// a wave that ends with such a sum makes its tiles again from s * q + b itself, in
+// the same order (no instruction more in the loop).
 //
 // Staging. Activations and weights both go from global memory to LDS by DMA
 // into rings of stages, the stage that a wave reads first waited for with one
@@ -192,6 +195,40 @@ __device__ __forceinline__ void store_tile(uint16_t* __restrict__ y, f32x4_t v, 
   }
 }
 
+// The sums of one tile and 16 activation rows again, without the scaled scales: the
+// same weights and the same order, so the same bits wherever those do not overflow.
+__device__ __forceinline__ f32x4_t plain_tile(const uint16_t* __restrict__ x, const uint8_t* __restrict__ packed,
+                                              int tile, int row, int K, int h_last) {
+  const int lane = threadIdx.x & 63, c = lane >> 4, i16 = lane & 15;
+  const uint16_t* xr = x + (size_t)row * K + 32 * c;
+  const uint8_t* rec = packed + (size_t)tile * (K / QG_SET) * QG_RECORD;
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+  for (int h = 0; h <= h_last; ++h) {
+    const uint8_t* r = rec + (size_t)(h >> 1) * QG_RECORD;
+    const u32x4 w = load16(r + (h & 1) * 512 + (c & 1) * 1024 + ((c >> 1) * 16 + i16) * 16);
+    const uint32_t sb = *reinterpret_cast<const uint32_t*>(r + QG_WBYTES + (h & 1) * 128 + ((c >> 1) * 16 + i16) * 4);
+    const float s = bf16_lo(sb), b = bf16_hi(sb);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] = cvt2(fmaf((float)(w[j] >> (4 * e) & 15u), s, b), fmaf((float)(w[j] >> (4 * e + 16) & 15u), s, b));
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[0], v[1], v[2], v[3]),
+                                                    __builtin_bit_cast(bf16x8_t, load16(xr + 128 * h + 8 * j)), acc, 0,
+                                                    0, 0);
+    }
+  }
+  return acc;
+}
+
+// v * 0 added: NaN from the first infinity or NaN on
+__device__ __forceinline__ void note_overflow(float& seen, f32x4_t v) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) seen = fmaf(v[r], 0.0f, seen);
+}
+
 // ---------------------------------------------------------------- 65 rows and more
 //
 // A block of NW waves owns 16 MT rows x 16 TPW NW outputs, wave w the weight
@@ -313,6 +350,20 @@ __global__ __launch_bounds__(64 * NW, PER_CU) void packed_gemm_kernel(const uint
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the LDS is given back with no DMA in flight
 
+  float seen = 0.0f;
+#pragma unroll
+  for (int p = 0; p < TPW; ++p)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) note_overflow(seen, acc[mt][p]);
+  if (__any(seen != 0.0f)) {
+#pragma unroll 1
+    for (int e = 0; e < TPW * MT; ++e) {
+      const int tile = tile0 + e / MT, m = m0 + 16 * (e % MT) + i16;
+      if (tile >= tiles) break;
+      store_tile<SWIGLU>(y, plain_tile(x, packed, tile, min(m, M - 1), K, h_last), tile, m, c, M, N, vec);
+    }
+    return;
+  }
 #pragma unroll
   for (int p = 0; p < TPW; ++p) {
     if (tile0 + p >= tiles) continue;
@@ -407,6 +458,16 @@ __global__ __launch_bounds__(256, 2) void packed_gemm_small_kernel(const uint16_
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (tile >= tiles) return;
+  float seen = 0.0f;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) note_overflow(seen, acc[mt]);
+  if (__any(seen != 0.0f)) {
+#pragma unroll 1
+    for (int mt = 0; mt < MT; ++mt)
+      store_tile<SWIGLU>(y, plain_tile(x, packed, tile, min(16 * mt + i16, M - 1), K, h_last), tile, 16 * mt + i16, c,
+                         M, N, vec);
+    return;
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) store_tile<SWIGLU>(y, acc[mt], tile, 16 * mt + i16, c, M, N, vec);
 }

@@ -66,3 +66,58 @@ def test_packed_gemm_swiglu_shapes(M, I):
     _C.call("qvex_swiglu", _ptr(gu), _ptr(h), M, I, _stream())
     torch.cuda.synchronize()
     assert torch.equal(fused.view(torch.int16), h.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(20, 100, 512), (64, 272, 1024), (70, 300, 512), (256, 6144, 256), (512, 24576, 256)])
+def test_packed_gemm_large_scales(M, N, K):
+    """Scales around 2^104 and of 2^116 (weights up to 2^120) beside ordinary ones: the
+    result is finite, within the bound of the shapes above, and a row without such a
+    scale has the bits it has alone. A scale that is infinite still gives what it is."""
+    w, s, b = synth.qmv_weights(N, K, seed=24)
+    s, b = synth.bf16_to_f32(s).copy(), synth.bf16_to_f32(b).copy()
+    plain = kernels.pack_w4(to_dev(w, torch.int32), to_dev(synth.bf16_bits(s), torch.bfloat16),
+                            to_dev(synth.bf16_bits(b), torch.bfloat16))
+    big = np.arange(3, N, 7)
+    for i, e in zip(range(4), (103, 104, 110, 116)):
+        rows = big[i::4]
+        s[rows, i % s.shape[1]] = np.float32(1.5 * 2.0 ** e)
+        b[rows, i % s.shape[1]] = np.float32(-8.0 * 1.5 * 2.0 ** e)
+    s16, b16 = synth.bf16_bits(s), synth.bf16_bits(b)
+    x = synth.qmv_x(M, K, seed=24)
+    xt = to_dev(x, torch.bfloat16)
+    y = kernels.packed_gemm(xt, kernels.pack_w4(to_dev(w, torch.int32), to_dev(s16, torch.bfloat16),
+                                                to_dev(b16, torch.bfloat16)), N)
+    torch.cuda.synchronize()
+    Wd = torch.from_numpy(synth.bf16_to_f32(_dequant_np(w, s16, b16)).astype(np.float64)).to(DEV)
+    xf = torch.from_numpy(synth.bf16_to_f32(x).astype(np.float64)).to(DEV)
+    ref = xf @ Wd.T
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -16 * (xf.abs() @ Wd.abs().T)
+    assert bool(y.isfinite().all())
+    assert bool(((y.double() - ref).abs() <= bound).all())
+    same = np.setdiff1d(np.arange(N), big)
+    assert torch.equal(y[:, same].view(torch.int16), kernels.packed_gemm(xt, plain, N)[:, same].view(torch.int16))
+    s[big[0], 0] = np.inf
+    y = kernels.packed_gemm(xt, kernels.pack_w4(to_dev(w, torch.int32), to_dev(synth.bf16_bits(s), torch.bfloat16),
+                                                to_dev(b16, torch.bfloat16)), N)
+    bad = ~y.isfinite()
+    assert bool(bad[:, big[0]].all())
+    bad[:, big[0]] = False
+    assert not bool(bad.any())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [40, 200])
+def test_packed_gemm_large_scales_swiglu(M):
+    K, I = 512, 520
+    w, s, b = synth.qmv_weights(2 * I, K, seed=25)
+    s, b = synth.bf16_to_f32(s).copy(), synth.bf16_to_f32(b).copy()
+    s[I + 5, 1], b[I + 5, 1] = 2.0 ** 110, -(2.0 ** 113)               # an up row
+    wt, st, bt = to_dev(w, torch.int32), to_dev(synth.bf16_bits(s), torch.bfloat16), to_dev(synth.bf16_bits(b), torch.bfloat16)
+    x = to_dev(synth.qmv_x(M, K, seed=25), torch.bfloat16)
+    fused = kernels.packed_gemm(x, kernels.pack_w4(wt, st, bt, swiglu=True), 2 * I, swiglu=True)
+    gu = kernels.packed_gemm(x, kernels.pack_w4(wt, st, bt), 2 * I)
+    h = torch.empty((M, I), dtype=torch.bfloat16, device=DEV)
+    _C.call("qvex_swiglu", _ptr(gu), _ptr(h), M, I, _stream())
+    torch.cuda.synchronize()
+    assert bool(fused.isfinite().all()) and torch.equal(fused.view(torch.int16), h.view(torch.int16))
