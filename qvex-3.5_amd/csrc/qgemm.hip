@@ -478,8 +478,9 @@ typedef void (*gemm_fn)(const uint16_t*, const uint8_t*, uint16_t*, int, int, in
 
 // The block shapes of packed_gemm_kernel, and what one round of blocks (as many
 // as the chip holds) takes relative to the others. Measured, K = 4096: 128 rows x
-// 384 outputs 97 us a round of 256, x 256 65 us, x 128 38 us, x 64 29 us, and
-// 64 rows x 64 outputs 28 us a round of 512 (20 us for 256 or fewer).
+// 384 outputs 97 us a round of 256, x 256 65 us, x 128 38 us, and 64 rows x 64
+// outputs 28 us a round of 512 (20 us for 256 or fewer; 128 x 64 took 29 us a round of
+// 256, never less than the 64 x 64 blocks of the same outputs).
 struct GemmShape {
   int rows, tiles;       // per block
   int threads;
@@ -492,8 +493,7 @@ struct GemmShape {
    {packed_gemm_kernel<MT, TPW, NW, AD, WD, PER_CU, false>, packed_gemm_kernel<MT, TPW, NW, AD, WD, PER_CU, true>}}
 const GemmShape kShapes[] = {
     GEMM_SHAPE(8, 3, 8, 3, 2, 1, 97.0f, 80.0f), GEMM_SHAPE(8, 2, 8, 3, 3, 1, 65.0f, 58.0f),
-    GEMM_SHAPE(8, 1, 8, 3, 3, 1, 38.0f, 37.0f), GEMM_SHAPE(8, 1, 4, 4, 4, 1, 29.0f, 29.0f),
-    GEMM_SHAPE(4, 1, 4, 3, 3, 2, 28.0f, 20.0f),
+    GEMM_SHAPE(8, 1, 8, 3, 3, 1, 38.0f, 37.0f), GEMM_SHAPE(4, 1, 4, 3, 3, 2, 28.0f, 20.0f),
 };
 
 // The shape whose rounds cost least: tall tiles of many outputs move the fewest

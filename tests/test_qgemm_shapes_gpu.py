@@ -1,8 +1,8 @@
 """Every block shape of the prefill GEMM at its edges (GPU): row counts around the
 16-row fragments, the small kernel's limit (64) and the row blocks (64, 128),
 output counts that end inside a tile, a wave or a column group (and, odd, take
-the element stores), the shortest K and ring wrap-arounds, and columns enough
-for each shape to be picked. Against x @ W~^T in float64, W~ the
+the element stores), the shortest K and ring wrap-arounds, and rows and columns
+that each shape is picked for. Against x @ W~^T in float64, W~ the
 bf16-dequantized weight: |y - ref| <= 2^-8 |ref| (the output's rounding) +
 2^-16 sum |x| |W~| (fp32 sums), as in tests/test_qgemm_gpu.py."""
 
@@ -17,7 +17,11 @@ from test_qmv_gpu import _dequant_np, to_dev
 
 SHAPES = [(16, 64, 256), (17, 301, 512), (32, 4097, 768), (33, 128, 2304), (48, 272, 1024), (49, 80, 256), (64, 65, 512),
           (65, 64, 256), (65, 16, 768), (100, 2049, 512), (127, 301, 256), (129, 1040, 1280), (130, 2048, 256),
-          (300, 4096, 512), (512, 8192, 256), (511, 10240, 768), (512, 24576, 256), (513, 12352, 512), (1000, 640, 2560)]
+          (300, 4096, 512), (512, 8192, 256), (511, 10240, 768), (512, 24576, 256), (513, 12352, 512), (1000, 640, 2560),
+          # 128 x 256 blocks (two tiles per wave): a partial row block, the columns ending in a wave's first tile
+          (129, 24592, 256), (200, 21861, 256),
+          # 128 x 384 blocks (three tiles per wave): the same, ending in a wave's first and second tile
+          (301, 24250, 256), (450, 24265, 256), (257, 24300, 512)]
 
 
 @pytest.mark.gpu
@@ -54,7 +58,9 @@ def test_packed_gemm_row_bits_over_shapes(N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,I", [(33, 264), (65, 512), (129, 1032), (512, 12288)])
+@pytest.mark.parametrize("M,I", [(33, 264), (65, 512), (129, 1032), (512, 12288),
+                                 # 128 x 128, 128 x 256 and 128 x 384 blocks, partial in rows and columns
+                                 (100, 8200), (130, 12296), (200, 12288), (301, 12136), (450, 12288)])
 def test_packed_gemm_swiglu_shapes(M, I):
     K = 512
     w, s, b = synth.qmv_weights(2 * I, K, seed=23, tag=M)
