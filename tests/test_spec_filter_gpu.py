@@ -350,3 +350,35 @@ def test_scores_kept_set_and_values(V, T, top_k, top_p, pen, bf16):
     ref = z[kept] - float(c0) - np.log(float(S))
     assert np.abs(got[kept] - ref).max() <= 1e-5 * (1.0 + np.abs(ref).max())
     print(f"V={V} top_k={top_k} top_p={top_p}: kept {int(kept.sum())}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [31, 32, 40])
+@pytest.mark.parametrize("k,V,T,top_k,top_p,pen,bf16,dl", [
+    (2, 8196, 0.7, 20, 0.9, 0.8, True, True),        # list filter, draft logits; V ends 4 past a part
+    (3, 12000, 1.0, 64, 1.0, 0.0, False, True),
+    (2, 8196, 0.8, 200, 0.95, 1.2, True, False),     # wide filter
+    (3, 16388, 0.9, 0, 0.9, 0.6, True, True),
+    (1, 8192, 1.2, 0, 0.8, 0.5, False, False),
+    (2, 20000, 0.7, 0, 1.0, 0.7, True, True),        # no filter, penalty
+    (0, 8196, 0.7, 300, 0.9, 0.4, True, False),
+    (2, 8196, 0.0, 0, 1.0, 0.9, True, False)])       # greedy
+def test_many_steps_bit_exact(S, k, V, T, top_k, top_p, pen, bf16, dl):
+    """Either side of the number of steps from which a step decides in a kernel of
+    its own and the weights are formed from its record, on every route that gets
+    there (draft logits or the wide filter), bf16 logits read as they are; the
+    penalty reaches the drafts before a row through the record."""
+    target, draft, ids, ua, us, seen = make_case(S, k, V, seed=S * 11 + k + V + top_k, bf16=bf16, draft_logits=dl)
+    t = torch.from_numpy(target).to(DEV)
+    if dl:
+        draft = synth.bf16_to_f32(synth.bf16_bits(draft)) if bf16 else draft
+    d = torch.from_numpy(draft).to(DEV) if dl else None
+    if bf16:
+        t, d = t.bfloat16(), d.bfloat16() if dl else None
+    sd = torch.from_numpy(seen).to(DEV)
+    kw = dict(presence_penalty=pen, top_k=top_k, top_p=top_p)
+    n, tok = kernels.spec_accept(t, d, torch.from_numpy(ids).to(DEV), torch.from_numpy(ua).to(DEV),
+                                 torch.from_numpy(us).to(DEV), T, seen=sd, **kw)
+    torch.cuda.synchronize()
+    n_o, tok_o = oracle.spec_accept(target, draft, ids, ua, us, inv(T), threads=16, seen=seen, **kw)
+    assert_same(n.cpu().numpy(), tok.cpu().numpy(), n_o, tok_o)
