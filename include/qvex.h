@@ -89,7 +89,8 @@ int qvex_qmv_affine(const uint16_t* x, const uint32_t* w, const uint16_t* scales
                     int group_size, void* stream);
 /* The same product for any M >= 1 (prompt chunks) on the matrix cores, from the
  * same layout: sum q*x and sum x per group in fp32, folded with the group's
- * scale and bias, one bf16 rounding. A row's result does not depend on M. */
+ * scale and bias, one bf16 rounding. A row's result does not depend on M; it can
+ * differ from qvex_qmv_affine's in the last bits (another order of the sums). */
 int qvex_affine_gemm(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
                      const uint16_t* biases, uint16_t* y, int M, int N, int K, int bits,
                      int group_size, void* stream);

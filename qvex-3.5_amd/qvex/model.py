@@ -151,7 +151,9 @@ class QLinear:
     it on chunks of 8 rows, so their rows have the same bits too; longer calls (prefill) run the packed
     MFMA GEMM (weights dequantized to bf16 in registers). Without a packed copy
     (K not a multiple of 256) the MLX-layout kernel takes calls, and chunks of
-    short tails, of 8 rows, and longer calls run qvex_affine_gemm."""
+    short tails, of 8 rows, and longer calls run qvex_affine_gemm; the two sum in
+    another order, so a row's bits differ between them, as they do between the
+    packed kernel and the packed GEMM, and are the same within each."""
 
     PACKED_MAX_ROWS = 8
     # calls of at least this many rows (prefill) run the packed GEMM; 0 disables it
@@ -204,6 +206,26 @@ class QLinear:
     def _packed_chunks(self, M: int) -> bool:
         """Rows for the packed kernel in chunks of PACKED_MAX_ROWS (below the dense GEMM)."""
         return self.packed is not None and M < max(self.DENSE_MIN_ROWS, self.PACKED_MAX_ROWS + 1)
+
+    def _chunks_beat_gemm(self, M: int) -> bool:
+        """Whether chunks of 8 rows finish before qvex_affine_gemm: a short call of a
+        long, narrow product, where the GEMM's time is its blocks' chain over K and a
+        chunk's is its weights (4 bits) or its waves' passes over K, 2048 codes each.
+        us, chunks | GEMM. 4 bits, 16 rows: 64 x 12352 13 | 49, 2048 x 8256 35 | 35,
+        4096 x 8256 61 | 34; 32 rows: 1024 x 12352 50 | 60, 1536 x 12352 73 | 60; 48 rows:
+        512 x 12352 45 | 60. Other widths, 16 rows: 1024 x 4096 at 3 bits, group 32 22 | 26, at
+        8 bits 20 | 19; 2048 x 8192 at 5 bits, group 32 39 | 45, at 6 bits, group 128 37 | 32;
+        1024 x 12352 at 8 bits 49 | 54; 24 rows of 1024 x 12288 at 3 bits, group 32 74 | 86, at 6 bits
+        75 | 79; 32 rows 97 | 87 and 100 | 79. Calls of 64 rows (a DeltaNet chunk) and more always
+        take the GEMM, so that a prompt's bits do not depend on how it is cut into such chunks."""
+        chunks = -(-M // QMV_MAX_ROWS)
+        if M >= 64:
+            return False
+        if (self.bits, self.group_size) == (4, 64):
+            return chunks * max(6.5, 1.0 + self.N * self.K / 2 ** 20) < self.K / 200
+        step = (2.7 if self.bits == 8 else 3.4) + {32: 2.0, 64: 1.4, 128: 0.4}[self.group_size]   # us per 1000 codes
+        gemm = 3.0 + step * self.K / 1000 * (1.0 if M <= 16 else 1.22)
+        return self.N <= 2048 and chunks * (2.5 + 3.9 * -(-self.K // 2048)) < gemm
 
     def swiglu(self, x) -> torch.Tensor:
         """silu(x W_gate^T) * (x W_up^T) for a fused [gate; up] layer
@@ -258,11 +280,8 @@ class QLinear:
             kernels.packed_gemm(x2.contiguous(), self.packed, self.N, out=o2)
             return out.view(*lead, self.N)
         w, sc, bi = self._mlx_on(x.device)
-        # two chunks of a long, narrow product finish before the GEMM's chain over K (16 rows of
-        # 512 x 12288: 42 us against 52; of 2048 x 4096: 30 against 24)
-        narrow = M <= 2 * QMV_MAX_ROWS and self.N <= 1024 and self.K >= 4096
         if self.packed is None and self.DENSE_MIN_ROWS and M >= max(self.DENSE_MIN_ROWS, QMV_MAX_ROWS + 1) \
-                and not narrow:
+                and not self._chunks_beat_gemm(M):
             kernels.quantized_matmul_affine(x2, w, sc, bi, self.group_size, self.bits, out=o2, gemm=True)
             return out.view(*lead, self.N)
         for m0 in range(0, M, QMV_MAX_ROWS):

@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from qvex import _C, kernels, synth
+from qvex.model import QLinear
 from test_affine_gpu import bits16, check, to_dev, weights
 
 
@@ -51,3 +52,27 @@ def test_affine_gemm_rejects(M, N, K, bits, gs):
     p16 = (ctypes.addressof(ctypes.create_string_buffer(64)) + 15) // 16 * 16
     with pytest.raises(_C.QvexError, match="qvex_affine_gemm"):
         _C.call("qvex_affine_gemm", p16, p16, p16, p16, p16, M, N, K, bits, gs, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,bits,gs,chunks", [
+    (16, 130, 8256, 4, 64, True), (48, 512, 12352, 4, 64, True), (40, 1024, 12352, 4, 64, False),
+    (63, 65, 12352, 4, 64, True), (64, 65, 12352, 4, 64, False), (16, 4096, 4160, 4, 64, False), (16, 130, 1088, 4, 64, False),
+    (16, 64, 8192, 5, 64, True), (17, 64, 8192, 5, 64, False), (16, 64, 8256, 8, 64, False), (16, 64, 12288, 8, 64, True),
+    (16, 2050, 8192, 6, 32, False), (24, 64, 12288, 3, 32, True), (32, 64, 12288, 3, 32, False), (15, 96, 448, 8, 64, True)])
+def test_unpacked_layer_takes_chunks_or_gemm(M, N, K, bits, gs, chunks):
+    """Either side of the rule that leaves a short call of a long, narrow layer to
+    chunks of 8 rows: the bits are those of the path it names, within the oracle's bound."""
+    w, s, b, _ = weights(N, K, bits, gs, seed=N + K)
+    x = synth.qmv_x(M, K, seed=23)
+    wt, st, bt = to_dev(w, torch.int32), to_dev(s, torch.bfloat16), to_dev(b, torch.bfloat16)
+    xt = to_dev(x, torch.bfloat16)
+    y = QLinear(wt, st, bt, gs, bits)(xt)
+    if chunks:
+        ref = torch.cat([kernels.quantized_matmul(xt[m:m + 8], wt, st, bt, group_size=gs, bits=bits)
+                         for m in range(0, M, 8)])
+    else:
+        ref = kernels.quantized_matmul_affine(xt, wt, st, bt, gs, bits, gemm=True)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+    check(x, w, s, b, bits, gs, bits16(y))
