@@ -154,10 +154,12 @@ __global__ __launch_bounds__(256) void conv_silu_qk_kernel(
 // flight together, the taps and the ring row are found once, and the window slides
 // through registers. The same operations in the same order per value: the same bits.
 // A wave per (token, head) spent its time on two 64-bit remainders, eight 2-byte tap
-// loads and one row's latency: 22.4 us for 512 tokens of 8192 channels (25 MB).
-// Now 9.2 us a call (10.4 with 16 tokens, 21.5 a token per wave); 1024 tokens 15.7
-// (39); up to 128 tokens the launch's 8 us, no slower at 9 tokens.
-constexpr int CONV_RUN = 8, CONV_RUN_MIN = 9;
+// loads and one row's latency: 21.7 us for 512 tokens of 8192 channels (25 MB).
+// Now 9.7 us a call (10.9 with 16 tokens); 1024 tokens 15.6 (39.7). A wave's eight tokens
+// are a longer chain, so calls whose blocks of a token per wave fit the chip at once
+// (4 per CU) keep those (us, token | run per wave): 9 tokens of 8192 channels 3.3 | 4.6,
+// 64 4.8 | 4.9, 100 6.4 | 5.2; 256 of 1024 3.7 | 4.7, 512 4.9 | 4.8; 64 of 4096 3.6 | 4.7, 256 7.0 | 5.2.
+constexpr int CONV_RUN = 8, CONV_RUN_BLOCKS = 1024;
 __global__ __launch_bounds__(256) void conv_silu_qk_run_kernel(
     const uint16_t* __restrict__ proj, long p_stride, uint16_t* __restrict__ ring, int R,
     const int32_t* __restrict__ pos, const uint16_t* __restrict__ cw, uint16_t* __restrict__ q,
@@ -1133,7 +1135,7 @@ extern "C" int qvex_gdn_conv_qk(const uint16_t* proj, long p_stride, uint16_t* c
                  "qvex_gdn_conv_qk: T=%d K=%d C=%d key_dim=%d Hv=%d", T, kernel_size, C, key_dim, Hv);
   QVEX_CHECK_ARG(ring_rows >= T + kernel_size - 1, "qvex_gdn_conv_qk: ring_rows=%d < T + K - 1 = %d", ring_rows,
                  T + kernel_size - 1);
-  if (kernel_size == 4 && T >= CONV_RUN_MIN)
+  if (kernel_size == 4 && (long)T * (C / 512) > CONV_RUN_BLOCKS)
     hipLaunchKernelGGL(conv_silu_qk_run_kernel, dim3((T + CONV_RUN - 1) / CONV_RUN, C / 512), dim3(256), 0,
                        (hipStream_t)stream, proj, p_stride, conv_ring, ring_rows, pos, conv_w, q, k, v, a_out, b_out,
                        T, C, key_dim, Hv, ab_offset, q_scale, k_scale, eps);
@@ -1205,7 +1207,6 @@ extern "C" int qvex_attn_qk_rope(const uint16_t* proj, long p_stride, const uint
 namespace {
 constexpr int ATT_ROWS = 16;
 constexpr int ATT_DSPLIT = 4;   // combine blocks per row, each over D / 4 dims (4 x the blocks in flight)
-
 }
 
 extern "C" uint64_t qvex_attn_workspace_bytes(int L, int Hq, int Hkv, int D, int max_keys, int keys_per_split) {

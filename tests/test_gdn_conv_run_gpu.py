@@ -1,7 +1,7 @@
-"""qvex_gdn_conv_qk on prompt chunks (8 consecutive tokens per wave) against the
-same tokens in calls of 8 or fewer (a token per wave): the same bits in q, k, v,
-a, b and in the ring, at partial runs, ring wrap-around and every position of the
-state rows."""
+"""qvex_gdn_conv_qk on prompt chunks (8 consecutive tokens per wave from 1024 blocks
+of 512 channels on, below that a token per wave) against the same tokens in calls
+of 8 or fewer: the same bits in q, k, v, a, b and in the ring, at partial runs, ring
+wrap-around and every position of the state rows."""
 
 import pytest
 import torch
@@ -26,6 +26,22 @@ def conv(proj, ring, pos, cw, C, key_dim, Hv, ab_off):
 @pytest.mark.parametrize("T,pos,spare", [(9, 0, 0), (15, 2, 1), (16, 1000, 0), (17, 14, 5), (40, 39, 0), (131, 7, 64)])
 @pytest.mark.parametrize("C,key_dim,Hv", [(1024, 256, 4), (1536, 128, 40)])
 def test_conv_runs_match_single_tokens(T, pos, spare, C, key_dim, Hv):
+    check(T, pos, spare, C, key_dim, Hv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,pos,spare", [(64, 5, 0), (65, 0, 0), (66, 68, 1), (71, 1000, 0), (72, 74, 5), (131, 7, 64)])
+def test_conv_runs_of_8_tokens_match_single_tokens(T, pos, spare):
+    """64 tokens of 8192 channels are the last call with a token per wave."""
+    check(T, pos, spare, 8192, 2048, 40)
+
+
+@pytest.mark.gpu
+def test_conv_runs_of_8_tokens_few_channels():
+    check(517, 3, 0, 1024, 256, 4)
+
+
+def check(T, pos, spare, C, key_dim, Hv):
     g = torch.Generator(device=DEV)
     g.manual_seed(T + pos)
     r = lambda *s: torch.randn(s, generator=g, device=DEV).bfloat16()
