@@ -216,16 +216,19 @@ class QLinear:
         512 x 12352 45 | 60. Other widths, 16 rows: 1024 x 4096 at 3 bits, group 32 22 | 26, at
         8 bits 20 | 19; 2048 x 8192 at 5 bits, group 32 39 | 45, at 6 bits, group 128 37 | 32;
         1024 x 12352 at 8 bits 49 | 54; 24 rows of 1024 x 12288 at 3 bits, group 32 74 | 86, at 6 bits
-        75 | 79; 32 rows 97 | 87 and 100 | 79. Calls of 64 rows (a DeltaNet chunk) and more always
+        75 | 79; 32 rows 97 | 87 and 100 | 79; a last chunk of one row takes 0.3 of a whole one (17
+        rows of 1024 x 12288 at 6 bits 59 | 79). Calls of 64 rows (a DeltaNet chunk) and more always
         take the GEMM, so that a prompt's bits do not depend on how it is cut into such chunks."""
-        chunks = -(-M // QMV_MAX_ROWS)
+        tail = M % QMV_MAX_ROWS
+        chunks = M // QMV_MAX_ROWS + (0.2 + 0.1 * tail if tail else 0.0)
         if M >= 64:
             return False
         if (self.bits, self.group_size) == (4, 64):
             return chunks * max(6.5, 1.0 + self.N * self.K / 2 ** 20) < self.K / 200
         step = (2.7 if self.bits == 8 else 3.4) + {32: 2.0, 64: 1.4, 128: 0.4}[self.group_size]   # us per 1000 codes
         gemm = 3.0 + step * self.K / 1000 * (1.0 if M <= 16 else 1.22)
-        return self.N <= 2048 and chunks * (2.5 + 3.9 * -(-self.K // 2048)) < gemm
+        a_pass = 3.4 if self.N <= 256 else 3.9
+        return self.N <= 2048 and chunks * (2.5 + a_pass * -(-self.K // 2048)) < gemm
 
     def swiglu(self, x) -> torch.Tensor:
         """silu(x W_gate^T) * (x W_up^T) for a fused [gate; up] layer

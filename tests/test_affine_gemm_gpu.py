@@ -58,7 +58,7 @@ def test_affine_gemm_rejects(M, N, K, bits, gs):
 @pytest.mark.parametrize("M,N,K,bits,gs,chunks", [
     (16, 130, 8256, 4, 64, True), (48, 512, 12352, 4, 64, True), (40, 1024, 12352, 4, 64, False),
     (63, 65, 12352, 4, 64, True), (64, 65, 12352, 4, 64, False), (16, 4096, 4160, 4, 64, False), (16, 130, 1088, 4, 64, False),
-    (16, 64, 8192, 5, 64, True), (17, 64, 8192, 5, 64, False), (16, 64, 8256, 8, 64, False), (16, 64, 12288, 8, 64, True),
+    (16, 512, 8192, 5, 64, True), (17, 512, 8192, 5, 64, True), (24, 512, 8192, 5, 64, False), (16, 64, 8256, 8, 64, False), (16, 64, 12288, 8, 64, True),
     (16, 2050, 8192, 6, 32, False), (24, 64, 12288, 3, 32, True), (32, 64, 12288, 3, 32, False), (15, 96, 448, 8, 64, True)])
 def test_unpacked_layer_takes_chunks_or_gemm(M, N, K, bits, gs, chunks):
     """Either side of the rule that leaves a short call of a long, narrow layer to
