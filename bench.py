@@ -332,7 +332,7 @@ def spec_config3(S=256, k=4, V=248320, temperature=0.7):
     acc = float(n.float().mean())
     del target, draft
     torch.cuda.empty_cache()
-    return {"kernel": "qvex_spec_accept (3 kernels: rowstats, decide, sample)", "steps": S, "k": k, "V": V,
+    return {"kernel": "qvex_spec_accept (4 kernels: rowstats, decide, weights, sample)", "steps": S, "k": k, "V": V,
             "inputs": f"synth.spec_inputs(range({S}), k={k}) (seed {synth.SEED_SPEC}, the tested inputs)",
             "us": round(us, 1), "us_per_step": round(us / S, 3), "GB/s": round(nbytes / (us * 1e-6) / 1e9, 1),
             "frac": round(nbytes / (us * 1e-6) / 1e9 / PEAK_HBM_GBS, 4), "bytes": nbytes,

@@ -24,6 +24,7 @@
 //     weight as 4-bit group-64 (codes widened to nibbles, a group-128 scale and
 //     bias repeated for both 64-code halves), so such layers run the packed
 //     MFMA products and every fused epilogue of the 4-bit path unchanged.
+#include "lds_dma.h"
 #include "qvex_common.h"
 
 namespace {
@@ -167,16 +168,11 @@ __global__ __launch_bounds__(256) void qmv_affine_kernel(const uint16_t* __restr
 // permute per group. Bound by issue: a step's extraction (12 VALU instructions
 // for 8 bits), 8 fmas per row tile and group, 2 MFMAs per row tile.
 // us, against chunks of 8 rows through the VALU kernel: 200 rows of 4096 x 4096 at
-// 8 bits 34 (368), 512 rows of 12288 x 4096 at 6 bits 158, 1024 rows of
-// 24576 x 4096 at 8 bits 506.
+// 8 bits 30.5 (368; replays of a graph 34.4), 512 rows of 12288 x 4096 at 6 bits 155,
+// 1024 rows of 24576 x 4096 at 8 bits 484.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-
-__device__ __forceinline__ int row_swizzle(int r) {
-  const int b = (r >> 2) & 3;                                   // b -> 0, 2, 3, 1
-  return ((((b << 1) & 3) ^ ((b >> 1) * 3)) << 2) | (r & 3);
-}
 
 // the 8 codes at bit `sh` (a multiple of 8) of the words (lo, hi), as bf16
 template <int BITS>
@@ -464,7 +460,7 @@ void launch_gemm_group(hipStream_t st, const uint16_t* x, const uint32_t* w, con
   };
   // Tall blocks extract each code for more rows; below AFF_GEMM_TALL of them the
   // chip is not full and shorter ones finish sooner (us, 8 bits, K = 4096, blocks of
-  // 64 | 32 rows: 64 x 4096 33 | 24, 200 x 4096 37 | 34, 512 x 4096 51 | 64,
+  // 64 | 32 rows: 64 x 4096 34 | 25, 200 x 4096 37 | 34, 512 x 4096 51 | 63,
   // 100 x 24576 65 | 86; 20 x 24576 at 5 bits, half of 64 rows empty, 49 | 38)
   if (M <= 16)
     go(affine_gemm_kernel<BITS, G32, 1>, 16);

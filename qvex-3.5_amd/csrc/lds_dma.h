@@ -1,5 +1,6 @@
-// DMA from global memory to LDS, written as asm: the compiler otherwise makes
-// LDS reads wait for DMAs into other parts of a ring (and drains all of them).
+// LDS staging: DMA from global memory, and the order of rows that are read as MFMA
+// operands. The DMA is asm since the compiler otherwise makes LDS reads wait for
+// DMAs into other parts of a ring (and drains all of them).
 #pragma once
 #include "qvex_common.h"
 
@@ -31,6 +32,14 @@ __device__ __forceinline__ void arrive() {
 
 __device__ __forceinline__ uint32_t lds_offset(void* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)p;
+}
+
+// Rows of 256 bytes in LDS with their 16-byte chunk ch at ch ^ row_swizzle(row): the 16
+// lanes that one pass of ds_read_b128 serves (0-3, 12-15 of one quarter, 4-11 of the
+// next) then hit 16 different bank groups.
+__device__ __forceinline__ int row_swizzle(int r) {
+  const int b = (r >> 2) & 3;                                   // b -> 0, 2, 3, 1
+  return ((((b << 1) & 3) ^ ((b >> 1) * 3)) << 2) | (r & 3);
 }
 
 }  // namespace

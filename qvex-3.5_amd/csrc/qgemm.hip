@@ -64,11 +64,6 @@ constexpr int QG_WSLOT = 1024 + 256;        // a tile's codes and (scale, bias) 
 typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ int row_swizzle(int r) {
-  const int b = (r >> 2) & 3;                                   // b -> 0, 2, 3, 1
-  return ((((b << 1) & 3) ^ ((b >> 1) * 3)) << 2) | (r & 3);
-}
-
 // the scale (for either code position) and bias of one weight row's group
 struct GroupScale {
   float s0, s1, b;

@@ -635,7 +635,8 @@ __device__ __forceinline__ void rowstats_block(const SpecArgs& a, int p, int row
 
 // LISTS: the form with the top-k lists (filt == 1). Without them a thread holds its
 // 32 logits and little else: 54 registers instead of 172, 9 waves on a SIMD instead
-// of 2, and 2304 rows of 248320 fp32 logits take 354 us (6.5 TB/s) instead of 516.
+// of 2, and 2304 rows of 248320 fp32 logits take 336 us (6.8 TB/s; 386 in the first
+// passes of a loop, before the clocks settle) instead of 516.
 template <bool BF, bool LISTS>
 __global__ __launch_bounds__(NT) void spec_rowstats_kernel(SpecArgs a) {
   rowstats_block<BF, LISTS>(a, blockIdx.x, blockIdx.y, true);
@@ -1195,8 +1196,8 @@ __device__ __forceinline__ void part_weights(const SpecArgs& a, const SpecWs& W,
 // steps (DECIDE_STEPS) one block per step decides (WEIGHTS false, grid 1 x steps) and
 // spec_weights_kernel makes the sums: a decision is a chain of dependent loads of
 // about 5 us, which 31 parts x 256 steps of blocks repeated in several rounds.
-// 256 steps of 248320 logits with draft rows: 12 + 121 us (189 in one kernel, 205
-// with a load per logit); 128 steps 265 -> 241 in all, 16 to 32 no difference, fewer
+// 256 steps of 248320 logits with draft rows: 10 + 90 us (12 + 121 in the first passes
+// of a loop, where one kernel took 189 and one with a load per logit 205); 128 steps 265 -> 241 in all, 16 to 32 no difference, fewer
 // a launch more.
 constexpr int DECIDE_STEPS = 32;
 template <bool WEIGHTS>

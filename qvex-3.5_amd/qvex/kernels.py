@@ -109,8 +109,8 @@ def quantized_matmul_affine(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
     _check(out, "out", torch.bfloat16)
     if out.numel() != M * N:
         raise _C.QvexError("out has the wrong size")
-    _C.call("qvex_affine_gemm" if gemm else "qvex_qmv_affine", _ptr(x2), _ptr(w), _ptr(scales), _ptr(biases), _ptr(out), M, N, K, bits,
-            group_size, _stream())
+    _C.call("qvex_affine_gemm" if gemm else "qvex_qmv_affine", _ptr(x2), _ptr(w), _ptr(scales), _ptr(biases),
+            _ptr(out), M, N, K, bits, group_size, _stream())
     return out
 
 
