@@ -130,3 +130,17 @@ def test_attention_workspace_serves_smaller_calls():
                     assert n >= last and n >= prev.get(keys, 0), (Hq, Hkv, D, kps, L, keys)
                     assert n <= Hkv * -(-L // QT) * -(-keys // (kps if L < 9 else min(kps, 256))) * 16 * (D + 2) * 4
                     prev[keys] = last = n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pos0,L", [(100, 40), (2011, 512)])
+def test_prefill_attention_nan_query_stays_in_its_row(pos0, L):
+    """A row of NaN scores is NaN as softmax attention has it, whatever unit it falls in;
+    its tile's other rows keep their bits."""
+    q, k, v, gate = inputs(L, 8, 8, 256, pos0, seed=7)
+    clean = attention(q, k, v, gate, pos0, 128)
+    q[19, 3, 5] = float("nan")
+    got = attention(q, k, v, gate, pos0, 128)
+    assert got[19, 3].isnan().all()
+    got[19, 3] = clean[19, 3]
+    assert torch.equal(got.view(torch.int16), clean.view(torch.int16))
